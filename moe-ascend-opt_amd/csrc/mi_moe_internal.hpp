@@ -151,7 +151,7 @@ inline bool w4_decode_fits(int H, int I, int K, size_t lds) {
 
 // W4A16 grouped GEMMs (sorted path): 64-row tiles staged with a 272-byte row
 // stride (256 B of a 128-group + 16 B that spread the rows over the LDS
-// banks), double-buffered, with the row sums and pair indices; gate_up takes
+// banks), double-buffered, with the row sums and a spare of 256 bytes; gate_up takes
 // kGemm13Blocks blocks of 4 slices, down kGemm2Quads quads of 64 rows of H,
 // and each stages the workgroup's metadata for all of K.
 constexpr int kGemmRowStride = 272;

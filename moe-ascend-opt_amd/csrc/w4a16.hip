@@ -310,12 +310,13 @@ void w4a16_down_token_kernel(const int32_t* ids, const uint16_t* act, const char
 // ================================================================ grouped GEMMs (sorted path)
 // Work item: a row tile (up to kGemmRows = 64 routed rows of one expert, from
 // the routing kernel's tile list) x a block of output rows (gate_up: 8 gate/up
-// slices; down: 4 quads of 64 rows), each wave owning 16-row weight tiles of
-// the block over all of K, so no cross-wave reduction.
-// Per 128-k group the workgroup stages the tile's activation rows (bf16, row
-// stride kGemmRowStride) and their sums into LDS, double-buffered with one
-// barrier per group; each wave holds its 16 weight rows of the group (16 B per
-// lane) in registers, and the next group's loads are issued before the
+// slices; down: 4 quads of 64 rows).  8 waves, each owning two 16-row weight
+// tiles of the block (gate and up of one slice; two row tiles of H) over all
+// of K, so no cross-wave reduction.
+// Per 128-k group the workgroup stages the tile's activation rows (row stride
+// kGemmRowStride) and their sums into LDS, double-buffered with one barrier
+// per group; each wave holds its weight rows of the group (16 B per lane and
+// tile) in registers, and the next group's loads are issued before the
 // current group is computed.  The workgroup's scales and zeros for all of K
 // (contiguous in the metadata layout) are copied into LDS once at the start,
 // so a step issues no per-lane metadata loads.  The MFMA A operand
@@ -327,26 +328,48 @@ void w4a16_down_token_kernel(const int32_t* ids, const uint16_t* act, const char
 // staged rows.  Every weight byte is read and dequantized once per
 // row tile, so an expert with many rows streams its weights a few times and
 // the MFMAs work on full 16-row operands.
+// What bounds them: the issue of dequantization, folds and LDS reads, which a
+// wave alone does not overlap with its MFMAs.  Two weight tiles per wave need
+// 124-128 VGPRs, so two workgroups (16 waves) share a CU; four tiles per wave
+// in 4-wave workgroups took 222-232 VGPRs and left 8 waves.
+// The results leave through the staging buffers, which are free by then: a
+// wave holds 16 columns (32 bytes) of a row, the workgroup 256 or 512 bytes of
+// it, and whole rows go out in 16-byte stores.  With 2-byte stores from the
+// registers the down GEMM spent about a quarter of its time on them.
+// Whole calls, H=2048 I=768 E=128 top-8, 4-wave form -> this one: T = 4096
+// 533 -> 488 us, Zipf-routed T = 512 134 -> 126 us, three layers at T = 37 258
+// -> 241 us; H=3072 I=1536 E=256: T = 64 327 -> 304 us, T = 1333 581 -> 549 us.
+// At T = 4096 the VALU is issued in 68% of the cycles, the matrix cores are
+// busy in 37%, and the clock drops to about 1.8 GHz.
 // LDS (kGemmLds, w4_gemm13_lds_bytes, w4_gemm2_lds_bytes): staged rows
-// [2][kGemmABytes] | row sums [2][kGemmRows] f32 | pair of each row
-// [kGemmRows] | the workgroup's metadata (gemm13: 4 * kGemm13Blocks slice
-// blocks of 80*G1 B; gemm2: 4 * kGemm2Quads sections of w2_meta_sec_bytes(G2) B)
+// [2][kGemmABytes], at the end the results | row sums [2][kGemmRows] f32 | a
+// spare [kGemmRows] f32 | the workgroup's metadata (gemm13: 4 * kGemm13Blocks
+// slice blocks of 80*G1 B; gemm2: 4 * kGemm2Quads sections of
+// w2_meta_sec_bytes(G2) B)
+constexpr int kGemmThreads = 512;
+static_assert(4 * kGemm13Blocks * kWave == kGemmThreads && 2 * kGemm2Quads * kWave == kGemmThreads,
+              "a slice, or two row tiles of H, per wave");
 
 // Copy nbytes (a multiple of 16) from global to LDS with the workgroup's
 // threads; the caller's barrier makes them visible.
 __device__ __forceinline__ void gemm_copy_meta(unsigned char* dst, const unsigned char* src, int nbytes, int tid) {
-  for (int k = tid; k < (nbytes >> 4); k += kBlock)
+  for (int k = tid; k < (nbytes >> 4); k += kGemmThreads)
     *reinterpret_cast<u32x4_t*>(dst + 16 * k) = ldg16(src + 16 * k);
 }
 
-// The staging thread's 32 values of its row (4 x 16 B) and their sum over the
-// row's 128 values (v_dot2 with (1, 1), then the row's 4 threads, which are
-// adjacent lanes).
+// acc of another lane of the row's 8 (a VALU lane move, no LDS round trip)
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+
+// The sum of a row's 128 values from the staging threads' 16 each (2 x 16 B):
+// v_dot2 with (1, 1), then over the row's 8 threads, which are adjacent lanes.
 template <int ACT>
-__device__ __forceinline__ float gemm_row_sum(const u32x4_t (&v)[4]) {
+__device__ __forceinline__ float gemm_row_sum(const u32x4_t (&v)[2]) {
   float acc = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < 2; ++i) {
     const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -358,17 +381,30 @@ __device__ __forceinline__ float gemm_row_sum(const u32x4_t (&v)[4]) {
                                      __builtin_bit_cast(f16x2_t, 0x3c003c00u), acc, false);
     }
   }
-  acc += __shfl_xor(acc, 1);
-  acc += __shfl_xor(acc, 2);
+  acc += dpp_f32<0xB1>(acc);    // quad_perm [1,0,3,2]
+  acc += dpp_f32<0x4E>(acc);    // quad_perm [2,3,0,1]
+  acc += dpp_f32<0x141>(acc);   // row_half_mirror: the other quad of 8 lanes
   return acc;
 }
 
 __device__ __forceinline__ void gemm_stage_store(unsigned char* buf, float* sums, int srow, int spart,
-                                                 const u32x4_t (&v)[4], float sum) {
-  unsigned char* d = buf + srow * kGemmRowStride + spart * 64;
+                                                 const u32x4_t (&v)[2], float sum) {
+  unsigned char* d = buf + srow * kGemmRowStride + spart * 16;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4_t*>(d + 16 * i) = v[i];
+  for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4_t*>(d + 128 * i) = v[i];
   if (spart == 0) sums[srow] = sum;
+}
+
+// A row's results, N * 128 bytes gathered in LDS by the waves of its 16-column
+// pieces, to global memory: N 16-byte stores per thread, 128 contiguous bytes
+// per row and instruction.
+constexpr int kGemm2OutStride = 128 * kGemm2Quads + 16;
+static_assert(kGemmRows * kGemm2OutStride <= 2 * kGemmABytes, "the down results fit the staging buffers");
+template <int N>
+__device__ __forceinline__ void gemm_store_row(uint16_t* dst, const unsigned char* src, int spart) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    *reinterpret_cast<u32x4_t*>(dst + 64 * i + 8 * spart) = lds16(src + 128 * i + 16 * spart);
 }
 
 // acc[p][s] += scale[p] * (W_p x - cz[p] * sum x) for the sub-tiles holding
@@ -400,11 +436,10 @@ __device__ __forceinline__ void gemm_group(const unsigned char* buf, const float
 }
 
 // gate_up + SiLU*mul: work item (row tile, kGemm13Blocks consecutive blocks of
-// 4 slices, a slice = 16 gate and 16 up rows); wave w owns slice w of each
-// block, so a staged activation row serves 2 * kGemm13Blocks weight tiles per
-// wave.  act[pair] gets the slices' 16 values each.
+// 4 slices, a slice = 16 gate and 16 up rows); wave w owns slice w of the
+// workgroup's 8.  act[pair] gets the slices' 16 values each.
 template <int ACT, int SDT>
-__global__ __launch_bounds__(kBlock) void w4a16_gemm13_kernel(const int32_t* ntiles, const int32_t* tiles,
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4))) void w4a16_gemm13_kernel(const int32_t* ntiles, const int32_t* tiles,
                                                              const int32_t* tok, const uint16_t* x, const void* w13,
                                                              const unsigned char* w13_m, int H_, int I_, W4Args a0) {
   // the leading arguments repeat fields of a0 (the first 14 dwords are
@@ -418,29 +453,29 @@ __global__ __launch_bounds__(kBlock) void w4a16_gemm13_kernel(const int32_t* nti
   a.w13_m = w13_m;
   a.c.H = H_;
   a.c.I = I_;
-  constexpr int NB = kGemm13Blocks;
+  constexpr int NB = 1;   // slices per wave
+  constexpr int NS = 4 * kGemm13Blocks;
   const SchedArgs& c = a.c;
   extern __shared__ __align__(16) unsigned char smem[];
-  const int H = c.H, NI1 = c.I >> 4, G1 = H >> 7, NSB = NI1 / (4 * NB);
+  const int H = c.H, NI1 = c.I >> 4, G1 = H >> 7, NSB = NI1 / NS;
   const int ti = blockIdx.x / NSB, sb = blockIdx.x - ti * NSB;
   if (ti >= *c.rg.ntiles) return;   // uniform
   const int4 tl = reinterpret_cast<const int4*>(c.rg.tiles)[ti];
   const int e = tl.x, row0 = tl.y, rows = tl.z, nsub = (rows + 15) >> 4;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, r = lane & 15;
-  const int srow = tid >> 2, spart = tid & 3;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, q = lane >> 4, r = lane & 15;
+  const int srow = tid >> 3, spart = tid & 7;
   const int spair = c.rg.tok[row0 + min(srow, rows - 1)];
-  const uint16_t* xsrc = c.x + (size_t)(spair / c.K) * H + 32 * spart;
+  const uint16_t* xsrc = c.x + (size_t)(spair / c.K) * H + 8 * spart;
   float* sums0 = reinterpret_cast<float*>(smem + 2 * kGemmABytes);
-  int* pairs = reinterpret_cast<int*>(sums0 + 2 * kGemmRows);   // the tile's pair indices
   unsigned char* meta = smem + kGemmLds;                         // [4 * NB slices][80 * G1]
-  gemm_copy_meta(meta, a.w13_m + ((size_t)e * NI1 + 4 * NB * sb) * 80 * G1, 4 * NB * 80 * G1, tid);
+  gemm_copy_meta(meta, a.w13_m + ((size_t)e * NI1 + NS * sb) * 80 * G1, NS * 80 * G1, tid);
   const char* wg[NB];
   const uint32_t* msc[NB];
   const unsigned char* mz[NB];
 #pragma unroll
   for (int p = 0; p < NB; ++p) {
-    const int jl = 4 * p + wave;   // slice within the workgroup's blocks
-    wg[p] = (const char*)a.w13 + ((size_t)e * NI1 + 4 * NB * sb + jl) * 2 * G1 * 1024 + lane * 16;
+    const int jl = 8 * p + wave;   // slice within the workgroup's blocks
+    wg[p] = (const char*)a.w13 + ((size_t)e * NI1 + NS * sb + jl) * 2 * G1 * 1024 + lane * 16;
     const unsigned char* mb = meta + jl * 80 * G1;
     msc[p] = reinterpret_cast<const uint32_t*>(mb) + r * G1;
     mz[p] = mb + 64 * G1 + r * G1;
@@ -449,17 +484,16 @@ __global__ __launch_bounds__(kBlock) void w4a16_gemm13_kernel(const int32_t* nti
 
   // only the waves of the sub-tiles holding rows store staged activations
   // (uniform per wave); every wave loads, so the loads stay unconditional
-  const bool stager = wave < nsub;
-  u32x4_t sv[4];
+  const bool stager = wave < 2 * nsub;
+  u32x4_t sv[2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) sv[i] = ldg16(xsrc + 8 * i);
+  for (int i = 0; i < 2; ++i) sv[i] = ldg16(xsrc + 64 * i);
   u32x4_t wc[2 * NB];
 #pragma unroll
   for (int p = 0; p < NB; ++p) {
     wc[2 * p] = ldg16(wg[p]);
     wc[2 * p + 1] = ldg16(wg[p] + (size_t)G1 * 1024);
   }
-  if (spart == 0) pairs[srow] = spair;
   if (stager) gemm_stage_store(smem, sums0, srow, spart, sv, gemm_row_sum<ACT>(sv));
   __syncthreads();
   f32x4_t acc[2 * NB][4];
@@ -473,7 +507,7 @@ __global__ __launch_bounds__(kBlock) void w4a16_gemm13_kernel(const int32_t* nti
     const int gn = more ? g + 1 : g;
     // next group: issued before this one is computed
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sv[i] = ldg16(xsrc + 128 * gn + 8 * i);
+    for (int i = 0; i < 2; ++i) sv[i] = ldg16(xsrc + 128 * gn + 64 * i);
     u32x4_t wn[2 * NB];
 #pragma unroll
     for (int p = 0; p < NB; ++p) {
@@ -513,26 +547,26 @@ __global__ __launch_bounds__(kBlock) void w4a16_gemm13_kernel(const int32_t* nti
       if (s < nsub) {
         const float gv[4] = {acc[2 * p][s].x, acc[2 * p][s].y, acc[2 * p][s].z, acc[2 * p][s].w};
         const float uv[4] = {acc[2 * p + 1][s].x, acc[2 * p + 1][s].y, acc[2 * p + 1][s].z, acc[2 * p + 1][s].w};
-        const int j = 4 * NB * sb + 4 * p + wave;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int row = 16 * s + 4 * q + v;
-          if (row < rows)
-            a.act[(size_t)pairs[row] * c.I + 16 * j + r] = from_f32<ACT>(silu_mul_fast(gv[v], uv[v]));
-        }
+        for (int v = 0; v < 4; ++v)
+          *reinterpret_cast<uint16_t*>(smem + (16 * s + 4 * q + v) * kGemmRowStride + 32 * (8 * p + wave) + 2 * r) =
+              from_f32<ACT>(silu_mul_fast(gv[v], uv[v]));
       }
     }
+  __syncthreads();
+  if (srow < rows)
+    gemm_store_row<2>(a.act + (size_t)spair * c.I + 16 * NS * sb, smem + srow * kGemmRowStride, spart);
 }
 
 // down: work item (row tile, kGemm2Quads consecutive quads m.. of H, a quad =
-// 64 rows); wave w owns the 16-row tile 64m + 16w of each quad, so a staged
-// activation row serves kGemm2Quads weight tiles (the rows are re-staged by
-// every workgroup of the tile: 2 quads halve that traffic).  eout[pair] gets
+// 64 rows); wave w owns 16-row tiles w and w + 8 of the workgroup's 16 (the
+// rows are re-staged by every workgroup of the tile: wider workgroups cut that
+// traffic).  eout[pair] gets
 // the tiles' values rounded to the activation dtype (the precision of the
 // act rows they come from; half the fp32 bytes written here and read by the
 // combine kernel, which sums over k in fp32).
 template <int ACT, int SDT>
-__global__ __launch_bounds__(kBlock) void w4a16_gemm2_kernel(const int32_t* ntiles, const int32_t* tiles,
+__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4))) void w4a16_gemm2_kernel(const int32_t* ntiles, const int32_t* tiles,
                                                             const int32_t* tok, const uint16_t* act, const void* w2,
                                                             const unsigned char* w2_m, int H_, int I_, W4Args a0) {
   // the leading arguments repeat fields of a0 (preloaded; see the gate_up GEMM)
@@ -553,37 +587,37 @@ __global__ __launch_bounds__(kBlock) void w4a16_gemm2_kernel(const int32_t* ntil
   if (ti >= *c.rg.ntiles) return;   // uniform
   const int4 tl = reinterpret_cast<const int4*>(c.rg.tiles)[ti];
   const int e = tl.x, row0 = tl.y, rows = tl.z, nsub = (rows + 15) >> 4;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, q = lane >> 4, r = lane & 15;
-  const int srow = tid >> 2, spart = tid & 3;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, q = lane >> 4, r = lane & 15;
+  const int srow = tid >> 3, spart = tid & 7;
   const int spair = c.rg.tok[row0 + min(srow, rows - 1)];
-  const uint16_t* asrc = a.act + (size_t)spair * I + 32 * spart;
-  const char* wb[kGemm2Quads];
-  const unsigned char* sec[kGemm2Quads];
+  const uint16_t* asrc = a.act + (size_t)spair * I + 8 * spart;
+  constexpr int NT = kGemm2Quads / 2;   // tiles per wave
+  const char* wb[NT];
+  const unsigned char* sec[NT];
   float* sums0 = reinterpret_cast<float*>(smem + 2 * kGemmABytes);
-  int* pairs = reinterpret_cast<int*>(sums0 + 2 * kGemmRows);
   unsigned char* meta = smem + kGemmLds;   // [kGemm2Quads quads][4 tiles][SEC], contiguous in HBM
   gemm_copy_meta(meta, a.w2_m + ((size_t)e * MQ + m0) * 4 * SEC, kGemm2Quads * 4 * SEC, tid);
 #pragma unroll
-  for (int p = 0; p < kGemm2Quads; ++p) {
-    const size_t tile = ((size_t)e * MQ + m0 + p) * 4 + wave;
+  for (int p = 0; p < NT; ++p) {
+    const int tl8 = 8 * p + wave;   // 16-row tile within the workgroup's quads
+    const size_t tile = ((size_t)e * MQ + m0) * 4 + tl8;
     wb[p] = (const char*)a.w2 + tile * G2 * 1024 + lane * 16;
-    sec[p] = meta + (p * 4 + wave) * SEC;
+    sec[p] = meta + tl8 * SEC;
   }
   constexpr float off = W4Consts<ACT>::offset;
 
-  const bool stager = wave < nsub;
-  u32x4_t sv[4];
+  const bool stager = wave < 2 * nsub;
+  u32x4_t sv[2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) sv[i] = ldg16(asrc + 8 * i);
-  u32x4_t wc[kGemm2Quads];
+  for (int i = 0; i < 2; ++i) sv[i] = ldg16(asrc + 64 * i);
+  u32x4_t wc[NT];
 #pragma unroll
-  for (int p = 0; p < kGemm2Quads; ++p) wc[p] = ldg16(wb[p]);
-  if (spart == 0) pairs[srow] = spair;
+  for (int p = 0; p < NT; ++p) wc[p] = ldg16(wb[p]);
   if (stager) gemm_stage_store(smem, sums0, srow, spart, sv, gemm_row_sum<ACT>(sv));
   __syncthreads();
-  f32x4_t acc[kGemm2Quads][4];
+  f32x4_t acc[NT][4];
 #pragma unroll
-  for (int p = 0; p < kGemm2Quads; ++p)
+  for (int p = 0; p < NT; ++p)
 #pragma unroll
     for (int s = 0; s < 4; ++s) acc[p][s] = f32x4_t{0, 0, 0, 0};
   for (int g2 = 0; g2 < G2; ++g2) {
@@ -591,45 +625,47 @@ __global__ __launch_bounds__(kBlock) void w4a16_gemm2_kernel(const int32_t* ntil
     const bool more = g2 + 1 < G2;   // uniform
     const int gn = more ? g2 + 1 : g2;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sv[i] = ldg16(asrc + 128 * gn + 8 * i);
-    u32x4_t wn[kGemm2Quads];
+    for (int i = 0; i < 2; ++i) sv[i] = ldg16(asrc + 128 * gn + 64 * i);
+    u32x4_t wn[NT];
 #pragma unroll
-    for (int p = 0; p < kGemm2Quads; ++p) wn[p] = ldg16(wb[p] + (size_t)gn * 1024);
+    for (int p = 0; p < NT; ++p) wn[p] = ldg16(wb[p] + (size_t)gn * 1024);
     {
-      u32x4_t B[kGemm2Quads][4];
-      float scp[kGemm2Quads], czp[kGemm2Quads];
+      u32x4_t B[NT][4];
+      float scp[NT], czp[NT];
 #pragma unroll
-      for (int p = 0; p < kGemm2Quads; ++p) {
+      for (int p = 0; p < NT; ++p) {
         const uint32_t w4[4] = {wc[p].x, wc[p].y, wc[p].z, wc[p].w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) B[p][i] = deq4<ACT>(w4[i]);
         scp[p] = scale_of<SDT>(reinterpret_cast<const uint16_t*>(sec[p])[16 * g2 + r]);
         czp[p] = off + w2_zero(sec[p], G2, g2, r);
       }
-      gemm_group<ACT, kGemm2Quads, false>(smem + b * kGemmABytes, sums0 + b * kGemmRows, nsub, q, r, B, scp,
+      gemm_group<ACT, NT, false>(smem + b * kGemmABytes, sums0 + b * kGemmRows, nsub, q, r, B, scp,
                                            czp, acc);
     }
     if (more && stager)
       gemm_stage_store(smem + (b ^ 1) * kGemmABytes, sums0 + (b ^ 1) * kGemmRows, srow, spart, sv,
                        gemm_row_sum<ACT>(sv));
 #pragma unroll
-    for (int p = 0; p < kGemm2Quads; ++p) wc[p] = wn[p];
+    for (int p = 0; p < NT; ++p) wc[p] = wn[p];
     __syncthreads();
   }
-  uint16_t* eout = reinterpret_cast<uint16_t*>(c.eout);
 #pragma unroll
-  for (int p = 0; p < kGemm2Quads; ++p)
+  for (int p = 0; p < NT; ++p)
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       if (s < nsub) {
         const float vv[4] = {acc[p][s].x, acc[p][s].y, acc[p][s].z, acc[p][s].w};
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int row = 16 * s + 4 * q + v;
-          if (row < rows) eout[(size_t)pairs[row] * H + 64 * (m0 + p) + 16 * wave + r] = from_f32<ACT>(vv[v]);
-        }
+        for (int v = 0; v < 4; ++v)
+          *reinterpret_cast<uint16_t*>(smem + (16 * s + 4 * q + v) * kGemm2OutStride + 32 * (8 * p + wave) + 2 * r) =
+              from_f32<ACT>(vv[v]);
       }
     }
+  __syncthreads();
+  if (srow < rows)
+    gemm_store_row<2 * NT>(reinterpret_cast<uint16_t*>(c.eout) + (size_t)spair * H + 64 * m0,
+                           smem + srow * kGemm2OutStride, spart);
 }
 
 template <int ACT, int SDT>
@@ -642,12 +678,12 @@ static hipError_t launch_gemm_t(const W4Args& a, int tiles_max, hipStream_t st, 
   if (lds2 > kMaxLds)
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(w4a16_gemm2_kernel<ACT, SDT>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds2);
-  hipLaunchKernelGGL((w4a16_gemm13_kernel<ACT, SDT>), dim3(g13), dim3(kBlock), lds13, st, a.c.rg.ntiles, a.c.rg.tiles,
+  hipLaunchKernelGGL((w4a16_gemm13_kernel<ACT, SDT>), dim3(g13), dim3(kGemmThreads), lds13, st, a.c.rg.ntiles, a.c.rg.tiles,
                      a.c.rg.tok, a.c.x, a.w13, a.w13_m, a.c.H, a.c.I, a);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   if (mid && (err = hipEventRecord(mid, st)) != hipSuccess) return err;
-  hipLaunchKernelGGL((w4a16_gemm2_kernel<ACT, SDT>), dim3(g2), dim3(kBlock), lds2, st, a.c.rg.ntiles, a.c.rg.tiles,
+  hipLaunchKernelGGL((w4a16_gemm2_kernel<ACT, SDT>), dim3(g2), dim3(kGemmThreads), lds2, st, a.c.rg.ntiles, a.c.rg.tiles,
                      a.c.rg.tok, (const uint16_t*)a.act, a.w2, a.w2_m, a.c.H, a.c.I, a);
   return hipGetLastError();
 }

@@ -60,6 +60,26 @@ def test_small_parity(cuda, small, T, K):
     assert max_rel_err(y, ref) <= TOL
 
 
+@pytest.mark.parametrize("adt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows", [1, 8, 15, 16, 17, 33, 48, 63, 64, 65, 127])
+def test_sorted_row_tile_edges(cuda, small, rows, adt):
+    """An expert with `rows` routed rows on the grouped GEMMs (its last row tile
+    partly filled; the other expert's 66 rows leave a tile of 2): staging, row
+    sums and the results' way out through LDS at the edges of sub-tiles and
+    tiles.  Bound as above; a row gone astray is off by its whole size."""
+    w, h = small
+    E, H, I = SMALL["E"], SMALL["H"], SMALL["I"]
+    T = rows + 66
+    g = torch.Generator().manual_seed(rows)
+    ids = torch.full((T, 1), 5, dtype=torch.int32)
+    ids[torch.randperm(T, generator=g)[:rows]] = 2
+    tw = torch.rand(T, 1, generator=g) + 0.5
+    x = torch.randn(T, H, generator=g).to(adt)
+    y = _run(h, x, ids, tw, cuda)
+    ref = _oracle(x, ids, tw, w, E, I, adt)
+    assert token_rel_err(y, ref) <= TOL
+
+
 @pytest.mark.parametrize("T,K", [(3, 10), (4, 16), (7, 10), (64, 1), (5, 7)])
 def test_decode_boundary_shapes(cuda, T, K):
     """Top-10 and top-16 at up to 64 routed pairs run the decode path (16

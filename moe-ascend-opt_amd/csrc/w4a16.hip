@@ -350,6 +350,23 @@ constexpr int kGemmThreads = 512;
 static_assert(4 * kGemm13Blocks * kWave == kGemmThreads && 2 * kGemm2Quads * kWave == kGemmThreads,
               "a slice, or two row tiles of H, per wave");
 
+// Work item of workgroup b, nb blocks of output rows per tile: returns the
+// tile.  Workgroups go round-robin over the 8 XCDs, so a tile's nb workgroups
+// are those of one XCD (b mod 8) in a row: they stage the same activation rows
+// through one L2.
+// Against tiles spread over the XCDs: H=2048 I=768 E=128 top-8, T = 37 (three
+// layers) 240.0 -> 236.9 us, T = 512 Zipf-routed 127.4 -> 125.3 us, T = 4096
+// 493 -> 485 us; H=3072 I=1536 E=256, T = 64 308.0 -> 303.4 us, T = 1333 553 ->
+// 547 us.
+// Dealing two or four consecutive tiles to an XCD in turn, for their shared
+// weights, measured the same at T = 4096 and 2-3% slower with few rows per
+// expert.
+__device__ __forceinline__ int gemm_item(int b, int nb, int& blk) {
+  const int p = b >> 3, t = p / nb;
+  blk = p - t * nb;
+  return 8 * t + (b & 7);
+}
+
 // Copy nbytes (a multiple of 16) from global to LDS with the workgroup's
 // threads; the caller's barrier makes them visible.
 __device__ __forceinline__ void gemm_copy_meta(unsigned char* dst, const unsigned char* src, int nbytes, int tid) {
@@ -458,7 +475,8 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   const SchedArgs& c = a.c;
   extern __shared__ __align__(16) unsigned char smem[];
   const int H = c.H, NI1 = c.I >> 4, G1 = H >> 7, NSB = NI1 / NS;
-  const int ti = blockIdx.x / NSB, sb = blockIdx.x - ti * NSB;
+  int sb;
+  const int ti = gemm_item(blockIdx.x, NSB, sb);
   if (ti >= *c.rg.ntiles) return;   // uniform
   const int4 tl = reinterpret_cast<const int4*>(c.rg.tiles)[ti];
   const int e = tl.x, row0 = tl.y, rows = tl.z, nsub = (rows + 15) >> 4;
@@ -583,7 +601,8 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   extern __shared__ __align__(16) unsigned char smem[];
   const int H = c.H, I = c.I, G2 = I >> 7, MQ = H >> 6, NMB = MQ / kGemm2Quads;
   const int SEC = w2_meta_sec_bytes(G2);
-  const int ti = blockIdx.x / NMB, m0 = (blockIdx.x - ti * NMB) * kGemm2Quads;
+  int mb;
+  const int ti = gemm_item(blockIdx.x, NMB, mb), m0 = mb * kGemm2Quads;
   if (ti >= *c.rg.ntiles) return;   // uniform
   const int4 tl = reinterpret_cast<const int4*>(c.rg.tiles)[ti];
   const int e = tl.x, row0 = tl.y, rows = tl.z, nsub = (rows + 15) >> 4;
@@ -670,6 +689,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
 
 template <int ACT, int SDT>
 static hipError_t launch_gemm_t(const W4Args& a, int tiles_max, hipStream_t st, hipEvent_t mid) {
+  tiles_max = (tiles_max + 7) & ~7;   // whole rounds over the XCDs (gemm_item)
   const int g13 = tiles_max * (a.c.I / 64 / kGemm13Blocks), g2 = tiles_max * (a.c.H / 64 / kGemm2Quads);
   const size_t lds13 = w4_gemm13_lds_bytes(a.c.H), lds2 = w4_gemm2_lds_bytes(a.c.I);
   if (lds13 > kMaxLds)

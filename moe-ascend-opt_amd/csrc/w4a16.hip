@@ -382,11 +382,9 @@ __device__ __forceinline__ float dpp_f32(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
-// The sum of a row's 128 values from the staging threads' 16 each (2 x 16 B):
-// v_dot2 with (1, 1), then over the row's 8 threads, which are adjacent lanes.
+// acc plus a thread's 16 values of a row (2 x 16 B), in order: v_dot2 with (1, 1)
 template <int ACT>
-__device__ __forceinline__ float gemm_row_sum(const u32x4_t (&v)[2]) {
-  float acc = 0.0f;
+__device__ __forceinline__ float gemm_chain(const u32x4_t (&v)[2], float acc) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
@@ -400,18 +398,34 @@ __device__ __forceinline__ float gemm_row_sum(const u32x4_t (&v)[2]) {
                                      __builtin_bit_cast(f16x2_t, 0x3c003c00u), acc, false);
     }
   }
-  acc += dpp_f32<0xB1>(acc);    // quad_perm [1,0,3,2]
-  acc += dpp_f32<0x4E>(acc);    // quad_perm [2,3,0,1]
-  acc += dpp_f32<0x141>(acc);   // row_half_mirror: the other quad of 8 lanes
+  return acc;
+}
+
+// The sum X of a row's 128 values, in lanes 5 and 7 of the row's 8 (adjacent
+// lanes, 16 values each): (s0 + s1) + (s2 + s3) of its quarters, each summed in
+// order, so an odd lane goes on from the even lane's sum (whose own second
+// chain is not used).  X is multiplied by offset + zero (1024 and more with
+// fp16), so the order of this sum decides which of two 16-bit neighbours a
+// result rounds to, and how much of small values survives beside outliers: it
+// is a fixed part of the results.  The idle half of the second chain costs
+// 2-3% at T = 4096 (450 -> 464 us, H=2048 I=768 E=128 top-8) against one chain
+// per thread over other quarters, whose results differ in about 1e-4; calls
+// of some dozens of tokens take the same time.
+template <int ACT>
+__device__ __forceinline__ float gemm_row_sum(const u32x4_t (&v)[2]) {
+  float acc = gemm_chain<ACT>(v, 0.0f);
+  acc = gemm_chain<ACT>(v, dpp_f32<0xA0>(acc));   // quad_perm [0,0,2,2]
+  acc += dpp_f32<0x4E>(acc);                      // quad_perm [2,3,0,1]
+  acc += dpp_f32<0x114>(acc);                     // row_shr:4: the other quad of 8 lanes
   return acc;
 }
 
 __device__ __forceinline__ void gemm_stage_store(unsigned char* buf, float* sums, int srow, int spart,
                                                  const u32x4_t (&v)[2], float sum) {
-  unsigned char* d = buf + srow * kGemmRowStride + spart * 16;
+  unsigned char* d = buf + srow * kGemmRowStride + spart * 32;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4_t*>(d + 128 * i) = v[i];
-  if (spart == 0) sums[srow] = sum;
+  for (int i = 0; i < 2; ++i) *reinterpret_cast<u32x4_t*>(d + 16 * i) = v[i];
+  if (spart == 7) sums[srow] = sum;
 }
 
 // A row's results, N * 128 bytes gathered in LDS by the waves of its 16-column
@@ -485,7 +499,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, q = lane >> 4, r = lane & 15;
   const int srow = tid >> 3, spart = tid & 7;
   const int spair = c.rg.tok[row0 + min(srow, rows - 1)];
-  const uint16_t* xsrc = c.x + (size_t)(spair / c.K) * H + 8 * spart;
+  const uint16_t* xsrc = c.x + (size_t)(spair / c.K) * H + 16 * spart;
   float* sums0 = reinterpret_cast<float*>(smem + 2 * kGemmABytes);
   unsigned char* meta = smem + kGemmLds;                         // [4 * NB slices][80 * G1]
   gemm_copy_meta(meta, a.w13_m + ((size_t)e * NI1 + NS * sb) * 80 * G1, NS * 80 * G1, tid);
@@ -507,7 +521,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   const bool stager = wave < 2 * nsub;
   u32x4_t sv[2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) sv[i] = ldg16(xsrc + 64 * i);
+  for (int i = 0; i < 2; ++i) sv[i] = ldg16(xsrc + 8 * i);
   u32x4_t wc[2 * NB];
 #pragma unroll
   for (int p = 0; p < NB; ++p) {
@@ -527,7 +541,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
     const int gn = more ? g + 1 : g;
     // next group: issued before this one is computed
 #pragma unroll
-    for (int i = 0; i < 2; ++i) sv[i] = ldg16(xsrc + 128 * gn + 64 * i);
+    for (int i = 0; i < 2; ++i) sv[i] = ldg16(xsrc + 128 * gn + 8 * i);
     {
       u32x4_t B[2 * NB][4];
       float sc[2 * NB], cz[2 * NB];
@@ -610,7 +624,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, q = lane >> 4, r = lane & 15;
   const int srow = tid >> 3, spart = tid & 7;
   const int spair = c.rg.tok[row0 + min(srow, rows - 1)];
-  const uint16_t* asrc = a.act + (size_t)spair * I + 8 * spart;
+  const uint16_t* asrc = a.act + (size_t)spair * I + 16 * spart;
   constexpr int NT = kGemm2Quads / 2;   // tiles per wave
   const char* wb[NT];
   const unsigned char* sec[NT];
@@ -629,7 +643,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   const bool stager = wave < 2 * nsub;
   u32x4_t sv[2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) sv[i] = ldg16(asrc + 64 * i);
+  for (int i = 0; i < 2; ++i) sv[i] = ldg16(asrc + 8 * i);
   u32x4_t wc[NT];
 #pragma unroll
   for (int p = 0; p < NT; ++p) wc[p] = ldg16(wb[p]);
@@ -645,7 +659,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
     const bool more = g2 + 1 < G2;   // uniform
     const int gn = more ? g2 + 1 : g2;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) sv[i] = ldg16(asrc + 128 * gn + 64 * i);
+    for (int i = 0; i < 2; ++i) sv[i] = ldg16(asrc + 128 * gn + 8 * i);
     {
       u32x4_t B[NT][4];
       float scp[NT], czp[NT];

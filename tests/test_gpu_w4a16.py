@@ -80,6 +80,31 @@ def test_sorted_row_tile_edges(cuda, small, rows, adt):
     assert token_rel_err(y, ref) <= TOL
 
 
+@pytest.mark.parametrize("adt", [torch.bfloat16, torch.float16])
+def test_sorted_row_sums_beside_outliers(cuda, adt):
+    """The grouped GEMMs' row sum of a 128-group adds the sums of its quarters,
+    (s0 + s1) + (s2 + s3), and is multiplied by 128 or 1024 plus the zero point.
+    Here s0 and s1 are +-2^15, which cancel (their weights are the same), and
+    the values of s2 and s3 are about 2^-5, of which fp32 keeps little beside
+    2^15 (half an ulp is 2^-9).  Only the first group holds values, so that
+    the oracle's sum is empty when it meets the outliers.  Bound as above;
+    summed beside an outlier, the result is off by more than its size."""
+    E, H, I, T = 8, 512, 256, 70
+    w = list(w4a16_random(E, H, I, seed=21))
+    w[2], w[5] = w[2] * 16, w[5] * 16
+    w[0][:, 32] = w[0][:, 0]
+    g = torch.Generator().manual_seed(21)
+    x = torch.zeros(T, H, dtype=adt)
+    x[:, 0] = torch.where(torch.rand(T, generator=g) < 0.5, -2.0**15, 2.0**15).to(adt)
+    x[:, 32] = -x[:, 0]
+    for k in (88, 120):
+        x[:, k:k + 8] = (torch.randn(T, 8, generator=g) / 32).to(adt)
+    ids = torch.randint(0, E, (T, 1), generator=g, dtype=torch.int32)
+    tw = torch.ones(T, 1)
+    y = _run(_handle(E, H, I, w, True, cuda), x, ids, tw, cuda)
+    assert token_rel_err(y, _oracle(x, ids, tw, w, E, I, adt)) <= TOL
+
+
 @pytest.mark.parametrize("T,K", [(3, 10), (4, 16), (7, 10), (64, 1), (5, 7)])
 def test_decode_boundary_shapes(cuda, T, K):
     """Top-10 and top-16 at up to 64 routed pairs run the decode path (16

@@ -43,6 +43,7 @@
 //     expert's rows), the grouped GEMMs gate_up (-> act) and down (-> eout),
 //     and the combine kernel.
 #pragma clang fp contract(off)
+#include "gemm_items.hpp"
 #include "mi_moe_device.hpp"
 #include "mi_moe_internal.hpp"
 #include "mi_moe_sched.hpp"
@@ -352,21 +353,33 @@ constexpr int kGemmThreads = 512;
 static_assert(4 * kGemm13Blocks * kWave == kGemmThreads && 2 * kGemm2Quads * kWave == kGemmThreads,
               "a slice, or two row tiles of H, per wave");
 
-// Work item of workgroup b, nb blocks of output rows per tile: returns the
-// tile.  Workgroups go round-robin over the 8 XCDs, so a tile's nb workgroups
-// are those of one XCD (b mod 8) in a row: they stage the same activation rows
-// through one L2.
-// Against tiles spread over the XCDs: H=2048 I=768 E=128 top-8, T = 37 (three
-// layers) 240.0 -> 236.9 us, T = 512 Zipf-routed 127.4 -> 125.3 us, T = 4096
-// 493 -> 485 us; H=3072 I=1536 E=256, T = 64 308.0 -> 303.4 us, T = 1333 553 ->
-// 547 us.
-// Dealing two or four consecutive tiles to an XCD in turn, for their shared
-// weights, measured the same at T = 4096 and 2-3% slower with few rows per
-// expert.
-__device__ __forceinline__ int gemm_item(int b, int nb, int& blk) {
-  const int p = b >> 3, t = p / nb;
-  blk = p - t * nb;
-  return 8 * t + (b & 7);
+// The row tile and the block of output rows (of nb) that this workgroup takes;
+// false if there is none.  A tile's nb workgroups stage the same activation
+// rows, so 8 tiles that take the same time go one to an XCD, through one L2;
+// other groups of 8 (fewer tiles, or unequal ones) are spread over the XCDs,
+// or those with a heavy tile would work on while the rest of the chip waits.
+// W4A16, us a layer, tiles always one to an XCD -> always spread -> this rule:
+// H=4096 I=14336 E=8 top-2, T = 100 Zipf-routed 330 -> 267 -> 273, T = 128
+// 257 -> 246 -> 249, T = 40 182 -> 200 -> 187; H=512 I=14336 E=3 top-2, T = 40
+// (3 tiles) 111 -> 104 -> 106; H=2048 I=1024 E=64 top-6, T = 64 51.6 -> 58.3 ->
+// 51.8; E=128 and E=256 the same as one to an XCD within 1%.
+struct GemmTile {
+  int e, row0, rows, blk;
+};
+__device__ __forceinline__ bool gemm_tile(const int32_t* tiles, unsigned ntiles, unsigned nb, GemmTile& t) {
+  const GemmItem spread = gemm_item(blockIdx.x, nb, false), own = gemm_item(blockIdx.x, nb, true);
+  const unsigned first = spread.tile & ~(kXcds - 1), last = min(first + kXcds, ntiles) - 1;
+  if (first >= ntiles) return false;   // uniform
+  const int4* d = reinterpret_cast<const int4*>(tiles);
+  // both candidates and the group's ends in one round of scalar loads: the
+  // empty asm keeps the compiler from waiting for them one after the other
+  int r0 = d[first].z, r7 = d[last].z;
+  int4 ds = d[min(spread.tile, last)], dn = d[min(own.tile, last)];
+  asm("" : "+s"(r0), "+s"(r7), "+s"(ds.x), "+s"(ds.y), "+s"(ds.z), "+s"(ds.w), "+s"(dn.x), "+s"(dn.y), "+s"(dn.z),
+      "+s"(dn.w));
+  const bool even = gemm_even(first, ntiles, (unsigned)(r0 + 15) >> 4, (unsigned)(r7 + 15) >> 4);
+  t = even ? GemmTile{dn.x, dn.y, dn.z, (int)own.blk} : GemmTile{ds.x, ds.y, ds.z, (int)spread.blk};
+  return even || spread.tile < ntiles;   // uniform
 }
 
 // Copy nbytes (a multiple of 16) from global to LDS with the workgroup's
@@ -491,11 +504,9 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   const SchedArgs& c = a.c;
   extern __shared__ __align__(16) unsigned char smem[];
   const int H = c.H, NI1 = c.I >> 4, G1 = H >> 7, NSB = NI1 / NS;
-  int sb;
-  const int ti = gemm_item(blockIdx.x, NSB, sb);
-  if (ti >= *c.rg.ntiles) return;   // uniform
-  const int4 tl = reinterpret_cast<const int4*>(c.rg.tiles)[ti];
-  const int e = tl.x, row0 = tl.y, rows = tl.z, nsub = (rows + 15) >> 4;
+  GemmTile tl;
+  if (!gemm_tile(c.rg.tiles, *c.rg.ntiles, NSB, tl)) return;   // uniform
+  const int e = tl.e, row0 = tl.row0, rows = tl.rows, sb = tl.blk, nsub = (rows + 15) >> 4;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, q = lane >> 4, r = lane & 15;
   const int srow = tid >> 3, spart = tid & 7;
   const int spair = c.rg.tok[row0 + min(srow, rows - 1)];
@@ -616,11 +627,9 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   extern __shared__ __align__(16) unsigned char smem[];
   const int H = c.H, I = c.I, G2 = I >> 7, MQ = H >> 6, NMB = MQ / kGemm2Quads;
   const int SEC = w2_meta_sec_bytes(G2);
-  int mb;
-  const int ti = gemm_item(blockIdx.x, NMB, mb), m0 = mb * kGemm2Quads;
-  if (ti >= *c.rg.ntiles) return;   // uniform
-  const int4 tl = reinterpret_cast<const int4*>(c.rg.tiles)[ti];
-  const int e = tl.x, row0 = tl.y, rows = tl.z, nsub = (rows + 15) >> 4;
+  GemmTile tl;
+  if (!gemm_tile(c.rg.tiles, *c.rg.ntiles, NMB, tl)) return;   // uniform
+  const int e = tl.e, row0 = tl.row0, rows = tl.rows, m0 = tl.blk * kGemm2Quads, nsub = (rows + 15) >> 4;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, q = lane >> 4, r = lane & 15;
   const int srow = tid >> 3, spart = tid & 7;
   const int spair = c.rg.tok[row0 + min(srow, rows - 1)];
@@ -703,7 +712,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
 
 template <int ACT, int SDT>
 static hipError_t launch_gemm_t(const W4Args& a, int tiles_max, hipStream_t st, hipEvent_t mid) {
-  tiles_max = (tiles_max + 7) & ~7;   // whole rounds over the XCDs (gemm_item)
+  tiles_max = (tiles_max + kXcds - 1) / kXcds * kXcds;   // whole groups (gemm_item)
   const int g13 = tiles_max * (a.c.I / 64 / kGemm13Blocks), g2 = tiles_max * (a.c.H / 64 / kGemm2Quads);
   const size_t lds13 = w4_gemm13_lds_bytes(a.c.H), lds2 = w4_gemm2_lds_bytes(a.c.I);
   if (lds13 > kMaxLds)

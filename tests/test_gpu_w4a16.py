@@ -80,6 +80,29 @@ def test_sorted_row_tile_edges(cuda, small, rows, adt):
     assert token_rel_err(y, ref) <= TOL
 
 
+@pytest.mark.parametrize("H,I", [(512, 128), (512, 384), (1536, 256)])
+@pytest.mark.parametrize("rows", [[10] * 8, [10] * 9, [64, 33, 20] + [10] * 5, [128] * 4 + [49] + [7] * 12,
+                                  [100] + [1] * 16, [70]])
+def test_sorted_tile_lists(cuda, rows, H, I):
+    """Lists of 2 to 21 row tiles, whole and partial groups of 8, of one and of
+    several sub-tile counts, at top-2: each tile's blocks of output rows are
+    dealt to the workgroups once.  I = 128 is one block of gate_up and one step
+    of the down loop, I = 384 and H = 1536 odd and other numbers of blocks.
+    Bound as above; a block left out leaves zeros or another call's rows."""
+    E = 20
+    w = w4a16_random(E, H, I, seed=H + I)
+    g = torch.Generator().manual_seed(len(rows))
+    experts = torch.randperm(E, generator=g)[:len(rows)]
+    ids = torch.cat([torch.full((r,), int(e)) for r, e in zip(rows, experts)])
+    if len(ids) % 2:
+        ids = torch.cat([ids, ids[:1]])
+    ids = ids[torch.randperm(len(ids), generator=g)].to(torch.int32).reshape(-1, 2)
+    tw = torch.rand(ids.shape, generator=g) + 0.5
+    x = torch.randn(len(ids), H, generator=g).to(torch.bfloat16)
+    y = _run(_handle(E, H, I, w, True, cuda), x, ids, tw, cuda)
+    assert token_rel_err(y, _oracle(x, ids, tw, w, E, I, torch.bfloat16)) <= TOL
+
+
 @pytest.mark.parametrize("adt", [torch.bfloat16, torch.float16])
 def test_sorted_row_sums_beside_outliers(cuda, adt):
     """The grouped GEMMs' row sum of a 128-group adds the sums of its quarters,

@@ -151,12 +151,12 @@ inline bool w4_decode_fits(int H, int I, int K, size_t lds) {
 
 // W4A16 grouped GEMMs (sorted path): 64-row tiles staged with a 272-byte row
 // stride (256 B of a 128-group + 16 B that spread the rows over the LDS
-// banks), double-buffered, with the row sums and a spare of 256 bytes; gate_up takes
-// kGemm13Blocks blocks of 4 slices, down kGemm2Quads quads of 64 rows of H,
-// and each stages the workgroup's metadata for all of K.
+// banks), double-buffered, with the row sums; gate_up takes kGemm13Blocks
+// blocks of 4 slices, down kGemm2Quads quads of 64 rows of H, and each stages
+// the workgroup's metadata for all of K.
 constexpr int kGemmRowStride = 272;
 constexpr int kGemmABytes = kGemmRows * kGemmRowStride;
-constexpr size_t kGemmLds = 2 * (size_t)kGemmABytes + 3 * kGemmRows * sizeof(float);
+constexpr size_t kGemmLds = 2 * (size_t)kGemmABytes + 2 * kGemmRows * sizeof(float);
 constexpr int kGemm13Blocks = 2;
 constexpr int kGemm2Quads = 4;
 inline size_t w4_gemm13_lds_bytes(int H) { return kGemmLds + (size_t)4 * kGemm13Blocks * 80 * (H >> 7); }

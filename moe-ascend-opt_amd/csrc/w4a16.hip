@@ -345,13 +345,13 @@ void w4a16_down_token_kernel(const int32_t* ids, const uint16_t* act, const char
 // At T = 4096 the VALU is issued in 68% of the cycles, the matrix cores are
 // busy in 37%, and the clock drops to about 1.8 GHz.
 // LDS (kGemmLds, w4_gemm13_lds_bytes, w4_gemm2_lds_bytes): staged rows
-// [2][kGemmABytes], at the end the results | row sums [2][kGemmRows] f32 | a
-// spare [kGemmRows] f32 | the workgroup's metadata (gemm13: 4 * kGemm13Blocks
-// slice blocks of 80*G1 B; gemm2: 4 * kGemm2Quads sections of
-// w2_meta_sec_bytes(G2) B)
-constexpr int kGemmThreads = 512;
-static_assert(4 * kGemm13Blocks * kWave == kGemmThreads && 2 * kGemm2Quads * kWave == kGemmThreads,
+// [2][kGemmABytes], at the end the results | row sums [2][kGemmRows] f32 | the
+// workgroup's metadata (gemm13: 4 * kGemm13Blocks slice blocks of 80*G1 B;
+// gemm2: 4 * kGemm2Quads sections of w2_meta_sec_bytes(G2) B)
+constexpr int kGemmWaves = 8, kGemmThreads = kGemmWaves * kWave;
+static_assert(4 * kGemm13Blocks == kGemmWaves && 4 * kGemm2Quads == 2 * kGemmWaves,
               "a slice, or two row tiles of H, per wave");
+static_assert(kGemmRows * 8 == kGemmThreads, "8 threads stage a row");
 
 // The row tile and the block of output rows (of nb) that this workgroup takes;
 // false if there is none.  A tile's nb workgroups stage the same activation
@@ -499,8 +499,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   a.w13_m = w13_m;
   a.c.H = H_;
   a.c.I = I_;
-  constexpr int NB = 1;   // slices per wave
-  constexpr int NS = 4 * kGemm13Blocks;
+  constexpr int NS = 4 * kGemm13Blocks;   // slices of a workgroup, one per wave
   const SchedArgs& c = a.c;
   extern __shared__ __align__(16) unsigned char smem[];
   const int H = c.H, NI1 = c.I >> 4, G1 = H >> 7, NSB = NI1 / NS;
@@ -512,19 +511,12 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   const int spair = c.rg.tok[row0 + min(srow, rows - 1)];
   const uint16_t* xsrc = c.x + (size_t)(spair / c.K) * H + 16 * spart;
   float* sums0 = reinterpret_cast<float*>(smem + 2 * kGemmABytes);
-  unsigned char* meta = smem + kGemmLds;                         // [4 * NB slices][80 * G1]
+  unsigned char* meta = smem + kGemmLds;   // [NS slices][80 * G1]
   gemm_copy_meta(meta, a.w13_m + ((size_t)e * NI1 + NS * sb) * 80 * G1, NS * 80 * G1, tid);
-  const char* wg[NB];
-  const uint32_t* msc[NB];
-  const unsigned char* mz[NB];
-#pragma unroll
-  for (int p = 0; p < NB; ++p) {
-    const int jl = 8 * p + wave;   // slice within the workgroup's blocks
-    wg[p] = (const char*)a.w13 + ((size_t)e * NI1 + NS * sb + jl) * 2 * G1 * 1024 + lane * 16;
-    const unsigned char* mb = meta + jl * 80 * G1;
-    msc[p] = reinterpret_cast<const uint32_t*>(mb) + r * G1;
-    mz[p] = mb + 64 * G1 + r * G1;
-  }
+  const char* wg = (const char*)a.w13 + ((size_t)e * NI1 + NS * sb + wave) * 2 * G1 * 1024 + lane * 16;
+  const unsigned char* mb = meta + wave * 80 * G1;
+  const uint32_t* msc = reinterpret_cast<const uint32_t*>(mb) + r * G1;
+  const unsigned char* mz = mb + 64 * G1 + r * G1;
   constexpr float off = W4Consts<ACT>::offset;
 
   // only the waves of the sub-tiles holding rows store staged activations
@@ -533,17 +525,12 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   u32x4_t sv[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) sv[i] = ldg16(xsrc + 8 * i);
-  u32x4_t wc[2 * NB];
-#pragma unroll
-  for (int p = 0; p < NB; ++p) {
-    wc[2 * p] = ldg16(wg[p]);
-    wc[2 * p + 1] = ldg16(wg[p] + (size_t)G1 * 1024);
-  }
+  u32x4_t wc[2] = {ldg16(wg), ldg16(wg + (size_t)G1 * 1024)};   // gate, up
   if (stager) gemm_stage_store(smem, sums0, srow, spart, sv, gemm_row_sum<ACT>(sv));
   __syncthreads();
-  f32x4_t acc[2 * NB][4];
+  f32x4_t acc[2][4];
 #pragma unroll
-  for (int p = 0; p < 2 * NB; ++p)
+  for (int p = 0; p < 2; ++p)
 #pragma unroll
     for (int s = 0; s < 4; ++s) acc[p][s] = f32x4_t{0, 0, 0, 0};
   for (int g = 0; g < G1; ++g) {
@@ -554,30 +541,21 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
 #pragma unroll
     for (int i = 0; i < 2; ++i) sv[i] = ldg16(xsrc + 128 * gn + 8 * i);
     {
-      u32x4_t B[2 * NB][4];
-      float sc[2 * NB], cz[2 * NB];
+      u32x4_t B[2][4];
 #pragma unroll
-      for (int p = 0; p < 2 * NB; ++p) {
+      for (int p = 0; p < 2; ++p) {
         const uint32_t w4[4] = {wc[p].x, wc[p].y, wc[p].z, wc[p].w};
 #pragma unroll
         for (int i = 0; i < 4; ++i) B[p][i] = deq4<ACT>(w4[i]);
       }
       issue_order_fence();
       // the next group's weights, into the registers just unpacked
-#pragma unroll
-      for (int p = 0; p < NB; ++p) {
-        wc[2 * p] = ldg16(wg[p] + (size_t)gn * 1024);
-        wc[2 * p + 1] = ldg16(wg[p] + (size_t)(G1 + gn) * 1024);
-      }
-#pragma unroll
-      for (int p = 0; p < NB; ++p) {
-        const uint32_t scc = msc[p][g], zzc = mz[p][g];
-        sc[2 * p] = scale_of<SDT>(scc & 0xffffu);
-        sc[2 * p + 1] = scale_of<SDT>(scc >> 16);
-        cz[2 * p] = off + (float)(zzc & 0xfu);
-        cz[2 * p + 1] = off + (float)((zzc >> 4) & 0xfu);
-      }
-      gemm_group<ACT, 2 * NB, true>(smem + b * kGemmABytes, sums0 + b * kGemmRows, nsub, q, r, B, sc, cz, acc);
+      wc[0] = ldg16(wg + (size_t)gn * 1024);
+      wc[1] = ldg16(wg + (size_t)(G1 + gn) * 1024);
+      const uint32_t scc = msc[g], zzc = mz[g];
+      const float sc[2] = {scale_of<SDT>(scc & 0xffffu), scale_of<SDT>(scc >> 16)};
+      const float cz[2] = {off + (float)(zzc & 0xfu), off + (float)((zzc >> 4) & 0xfu)};
+      gemm_group<ACT, 2, true>(smem + b * kGemmABytes, sums0 + b * kGemmRows, nsub, q, r, B, sc, cz, acc);
     }
     if (more && stager)
       gemm_stage_store(smem + (b ^ 1) * kGemmABytes, sums0 + (b ^ 1) * kGemmRows, srow, spart, sv,
@@ -585,18 +563,16 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
     __syncthreads();
   }
 #pragma unroll
-  for (int p = 0; p < NB; ++p)
+  for (int s = 0; s < 4; ++s) {
+    if (s < nsub) {
+      const float gv[4] = {acc[0][s].x, acc[0][s].y, acc[0][s].z, acc[0][s].w};
+      const float uv[4] = {acc[1][s].x, acc[1][s].y, acc[1][s].z, acc[1][s].w};
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      if (s < nsub) {
-        const float gv[4] = {acc[2 * p][s].x, acc[2 * p][s].y, acc[2 * p][s].z, acc[2 * p][s].w};
-        const float uv[4] = {acc[2 * p + 1][s].x, acc[2 * p + 1][s].y, acc[2 * p + 1][s].z, acc[2 * p + 1][s].w};
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          *reinterpret_cast<uint16_t*>(smem + (16 * s + 4 * q + v) * kGemmRowStride + 32 * (8 * p + wave) + 2 * r) =
-              from_f32<ACT>(silu_mul_fast(gv[v], uv[v]));
-      }
+      for (int v = 0; v < 4; ++v)
+        *reinterpret_cast<uint16_t*>(smem + (16 * s + 4 * q + v) * kGemmRowStride + 32 * wave + 2 * r) =
+            from_f32<ACT>(silu_mul_fast(gv[v], uv[v]));
     }
+  }
   __syncthreads();
   if (srow < rows)
     gemm_store_row<2>(a.act + (size_t)spair * c.I + 16 * NS * sb, smem + srow * kGemmRowStride, spart);
@@ -634,7 +610,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   const int srow = tid >> 3, spart = tid & 7;
   const int spair = c.rg.tok[row0 + min(srow, rows - 1)];
   const uint16_t* asrc = a.act + (size_t)spair * I + 16 * spart;
-  constexpr int NT = kGemm2Quads / 2;   // tiles per wave
+  constexpr int NT = 4 * kGemm2Quads / kGemmWaves;   // tiles per wave
   const char* wb[NT];
   const unsigned char* sec[NT];
   float* sums0 = reinterpret_cast<float*>(smem + 2 * kGemmABytes);
@@ -642,10 +618,9 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
   gemm_copy_meta(meta, a.w2_m + ((size_t)e * MQ + m0) * 4 * SEC, kGemm2Quads * 4 * SEC, tid);
 #pragma unroll
   for (int p = 0; p < NT; ++p) {
-    const int tl8 = 8 * p + wave;   // 16-row tile within the workgroup's quads
-    const size_t tile = ((size_t)e * MQ + m0) * 4 + tl8;
-    wb[p] = (const char*)a.w2 + tile * G2 * 1024 + lane * 16;
-    sec[p] = meta + tl8 * SEC;
+    const int wt = kGemmWaves * p + wave;   // 16-row tile within the workgroup's quads
+    wb[p] = (const char*)a.w2 + (((size_t)e * MQ + m0) * 4 + wt) * G2 * 1024 + lane * 16;
+    sec[p] = meta + wt * SEC;
   }
   constexpr float off = W4Consts<ACT>::offset;
 
@@ -700,7 +675,7 @@ __global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4)
         const float vv[4] = {acc[p][s].x, acc[p][s].y, acc[p][s].z, acc[p][s].w};
 #pragma unroll
         for (int v = 0; v < 4; ++v)
-          *reinterpret_cast<uint16_t*>(smem + (16 * s + 4 * q + v) * kGemm2OutStride + 32 * (8 * p + wave) + 2 * r) =
+          *reinterpret_cast<uint16_t*>(smem + (16 * s + 4 * q + v) * kGemm2OutStride + 32 * (kGemmWaves * p + wave) + 2 * r) =
               from_f32<ACT>(vv[v]);
       }
     }

@@ -401,11 +401,11 @@ def _device_lds():
 @pytest.mark.parametrize("T,K", [(1, 2), (3, 2), (40, 2)])
 def test_large_intermediate_parity(cuda, T, K):
     """Mixtral-like I = 14336: the decode down kernel needs 66,440 B of LDS at
-    K = 2 and the sorted down GEMM 107,264 B.  Calls take the decode path where
+    K = 2 and the sorted down GEMM 107,008 B.  Calls take the decode path where
     it fits, else the sorted path; a handle is refused only if the sorted GEMMs
     exceed the device's LDS (checked at create, status 3)."""
     E, H, I = 3, 512, 14336
-    need_sorted = 2 * 64 * 272 + 3 * 64 * 4 + 16 * ((40 * (I // 128) + 15) & ~15)
+    need_sorted = 2 * 64 * 272 + 2 * 64 * 4 + 16 * ((40 * (I // 128) + 15) & ~15)
     w = w4a16_random(E, H, I, seed=77 + T)
     if need_sorted > _device_lds():
         with pytest.raises(RuntimeError, match="status 3"):

@@ -320,10 +320,10 @@ void w4a16_down_token_kernel(const int32_t* ids, const uint16_t* act, const char
 // tile) in registers, and the next group's loads are issued before the
 // current group's MFMAs, into the registers that the dequantization has just
 // read (a second set cost 8 register moves a step: T = 37 x 3 layers 236.7 ->
-// 233.0 us, Zipf-routed T = 512 128.0 -> 124.7 us, the rest within 1.5%).  The workgroup's scales and zeros for all of K
-// (contiguous in the metadata layout) are copied into LDS once at the start,
-// so a step issues no per-lane metadata loads.  The MFMA A operand
-// is 16 rows of the tile (sub-tiles of 16 rows; only the sub-tiles holding
+// 233.0 us, Zipf-routed T = 512 128.0 -> 124.7 us, the rest within 1.5%).  The
+// workgroup's scales and zeros for all of K (contiguous in the metadata layout)
+// are copied into LDS once at the start, so a step issues no per-lane metadata
+// loads.  The MFMA A operand is 16 rows of the tile (sub-tiles of 16 rows; only the sub-tiles holding
 // rows are computed), B the dequantized weights:
 //   acc += s * (sum_k x (magic + q) - (offset + z) * sum_k x)   per group,
 // the same arithmetic as the decode kernels, with the row sums from v_dot2
@@ -337,13 +337,13 @@ void w4a16_down_token_kernel(const int32_t* ids, const uint16_t* act, const char
 // in 4-wave workgroups took 222-232 VGPRs and left 8 waves.
 // The results leave through the staging buffers, which are free by then: a
 // wave holds 16 columns (32 bytes) of a row, the workgroup 256 or 512 bytes of
-// it, and whole rows go out in 16-byte stores.  With 2-byte stores from the
-// registers the down GEMM spent about a quarter of its time on them.
+// it, and whole rows go out in 16-byte stores (T = 4096: the down GEMM took 213
+// us with 2-byte stores from the registers, 190 with these, 153 with none).
 // Whole calls, H=2048 I=768 E=128 top-8, 4-wave form -> this one: T = 4096
-// 533 -> 488 us, Zipf-routed T = 512 134 -> 126 us, three layers at T = 37 258
-// -> 241 us; H=3072 I=1536 E=256: T = 64 327 -> 304 us, T = 1333 581 -> 549 us.
-// At T = 4096 the VALU is issued in 68% of the cycles, the matrix cores are
-// busy in 37%, and the clock drops to about 1.8 GHz.
+// 508 -> 454 us, Zipf-routed T = 512 125 -> 117 us, three layers at T = 37 258
+// -> 233 us; H=3072 I=1536 E=256: T = 64 323 -> 298 us, T = 1333 576 -> 537 us.
+// At T = 4096 gate_up issues VALU in 67% of the cycles and keeps the matrix
+// cores busy in 39% (down 66% and 31%).
 // LDS (kGemmLds, w4_gemm13_lds_bytes, w4_gemm2_lds_bytes): staged rows
 // [2][kGemmABytes], at the end the results | row sums [2][kGemmRows] f32 | the
 // workgroup's metadata (gemm13: 4 * kGemm13Blocks slice blocks of 80*G1 B;
@@ -359,8 +359,8 @@ static_assert(kGemmRows * 8 == kGemmThreads, "8 threads stage a row");
 // other groups of 8 (fewer tiles, or unequal ones) are spread over the XCDs,
 // or those with a heavy tile would work on while the rest of the chip waits.
 // W4A16, us a layer, tiles always one to an XCD -> always spread -> this rule:
-// H=4096 I=14336 E=8 top-2, T = 100 Zipf-routed 330 -> 267 -> 273, T = 128
-// 257 -> 246 -> 249, T = 40 182 -> 200 -> 187; H=512 I=14336 E=3 top-2, T = 40
+// H=4096 I=14336 E=8 top-2, T = 100 Zipf-routed 335 -> 268 -> 273, T = 128
+// 257 -> 246 -> 250, T = 40 182 -> 200 -> 187; H=512 I=14336 E=3 top-2, T = 40
 // (3 tiles) 111 -> 104 -> 106; H=2048 I=1024 E=64 top-6, T = 64 51.6 -> 58.3 ->
 // 51.8; E=128 and E=256 the same as one to an XCD within 1%.
 struct GemmTile {
